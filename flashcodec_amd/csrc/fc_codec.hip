@@ -140,17 +140,16 @@ __global__ __launch_bounds__(kThreads) void jpeg_decode_kernel(
     const TI* __restrict__ store, const float* __restrict__ scales, int64_t H, int64_t cap,
     int64_t a, int64_t nblk, int64_t D, int r, int k, const float* __restrict__ basis,
     TO* __restrict__ out, int64_t osb, int64_t osh, int64_t oss, int64_t out_len,
-    int64_t items, int lpi_log2, TailRows tail, int group = 0) {
+    int64_t items, int lpi_log2, int group = 0) {
   const ItemMap im = item_of_thread(lpi_log2);
   if (im.item >= items) return;
-  const int64_t bh = im.item / nblk, rel = im.item - bh * nblk, blk = a + rel;
+  const int64_t bh = im.item / nblk, blk = a + (im.item - bh * nblk);
   const int64_t b = bh / H, h = bh - b * H;
   const int64_t d0 = (int64_t)im.lane * VEC;
   if (d0 >= D) return;
   const int64_t row0 = (bh * cap + blk) * k;
   TO* dst = out + b * osb + h * osh + d0;
   const int64_t tok0 = blk * r;
-  if (rel == tail.at) return copy_tail<TO, VEC>(tail, b, h, d0, dst, tok0, oss);
 
   if constexpr (RMAX > 0) {
     float acc[RMAX][VEC];
@@ -679,9 +678,10 @@ static int jpeg_encode_launch(const void* x, int x_dtype, int64_t B, int64_t H, 
   const int fv = jpeg_vec_fast(x_dtype, pick_vec(D, 8, {x_sb, x_sh, x_ss},
                                                  {{x, es}, {coeffs, quant_bits ? 1 : es}}), D);
   if (jpeg_encode_fast_supported(r, x_dtype, fv, mode, s_valid >= m * r, gate != nullptr)) {
-    const int rc = jpeg_encode_fast(JpegEncodeLaunch{
-        x, x_dtype, x_sb, x_sh, x_ss, H, m, D, s_valid, r, k, basis, coeffs, scales, cap, n0,
-        items, log2_lanes(D, fv), fv, mode, gate, st});
+    const JpegEncodeArgs p{x_sb, x_sh, x_ss, H, m, D, s_valid, cap, n0, items, k,
+                           log2_lanes(D, fv)};
+    const int rc = jpeg_encode_fast(
+        JpegEncodeLaunch{p, x, x_dtype, r, basis, coeffs, scales, fv, mode, gate, st});
     return rc != FC_OK ? rc : check_launch();
   }
   const int lg = log2_lanes(D, vec);
@@ -813,7 +813,6 @@ static int jpeg_decode_launch(const void* store, int store_dtype, const float* s
       k > r)
     return FC_ERR_ARG;
   if (group && (group != 32 || store_dtype != FC_I8 || D % group)) return FC_ERR_ARG;
-  if (tail.n) tail.at = nblk;
   const int64_t nper = nblk + (tail.n ? 1 : 0);  // items per sequence
   const int64_t items = B * H * nper;
   if (items == 0) return FC_OK;
@@ -825,23 +824,30 @@ static int jpeg_decode_launch(const void* store, int store_dtype, const float* s
   if (!es_in || !es_out || out_dtype == FC_I8) return FC_ERR_ARG;
   const int rmax = rmax_for(r);
   const int vec =
-      pick_vec(D, max_vec_for(rmax), {o_sb, o_sh, o_ss, tail.sb, tail.sh, tail.st},
-               {{store, es_in}, {out, es_out}, {tail.p, es_out}});
+      pick_vec(D, max_vec_for(rmax), {o_sb, o_sh, o_ss}, {{store, es_in}, {out, es_out}});
   if (!vec) return FC_ERR_UNSUPPORTED;
   if (!quant && out_dtype != FC_F32 && out_dtype != store_dtype) return FC_ERR_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
   const int fv = jpeg_vec_fast(
-      out_dtype, pick_vec(D, 8, {o_sb, o_sh, o_ss, tail.sb, tail.sh, tail.st},
+      out_dtype, pick_vec(D, 8, {o_sb, o_sh, o_ss, tail.sb, tail.sh},
                           {{store, es_in}, {out, es_out}, {tail.p, es_out}}), D);
   const JpegMode mode = !quant ? kJpegFp : group ? kJpegGroup : kJpegRow;
-  if (jpeg_decode_fast_supported(k, out_dtype, fv, mode)) {
-    const int rc = jpeg_decode_fast(JpegDecodeLaunch{
-        store, store_dtype, out_dtype, scales, H, cap, a, nper, D, r, k, basis, out, o_sb, o_sh,
-        o_ss, out_len, items, log2_lanes(D, fv), fv, mode, tail, st});
+  if (jpeg_decode_fast_supported(r, k, out_dtype, fv, mode)) {
+    const JpegDecodeArgs p{H, cap, a, nper, D, o_sb, o_sh, o_ss, out_len, items, r, k,
+                           log2_lanes(D, fv)};
+    const int rc = jpeg_decode_fast(
+        JpegDecodeLaunch{p, store, store_dtype, out_dtype, scales, basis, out, fv, mode, tail, st});
     return rc != FC_OK ? rc : check_launch();
   }
+  if (tail.n) {  // behind the blocks, by the copy kernel
+    const int rc = fc_gather_segments(
+        static_cast<char*>(out) + (a + nblk) * r * o_ss * es_out, o_sb * es_out, o_sh * es_out,
+        tail.p, tail.sb * es_out, tail.sh * es_out, nullptr, B, B, H, tail.n * D * es_out, stream);
+    if (rc != FC_OK || nblk == 0) return rc;
+  }
   const int lg = log2_lanes(D, vec);
-  const dim3 grid = grid_for(items, lg);
+  const int64_t nitems = B * H * nblk;
+  const dim3 grid = grid_for(nitems, lg);
   auto launch = [&](auto ti, auto to) {
     using TI = decltype(ti);
     using TO = decltype(to);
@@ -850,9 +856,9 @@ static int jpeg_decode_launch(const void* store, int store_dtype, const float* s
       return with_int<8, 16, 0>(rmax, [&](auto rc_) {
         constexpr int RMAX = decltype(rc_)::value;
         jpeg_decode_kernel<TI, TO, VEC, RMAX, std::is_same<TI, int8_t>::value>
-            <<<grid, kThreads, 0, st>>>((const TI*)store, scales, H, cap, a, nper, D, r, k,
-                                        basis, (TO*)out, o_sb, o_sh, o_ss, out_len, items, lg,
-                                        tail, group);
+            <<<grid, kThreads, 0, st>>>((const TI*)store, scales, H, cap, a, nblk, D, r, k,
+                                        basis, (TO*)out, o_sb, o_sh, o_ss, out_len, nitems, lg,
+                                        group);
         return FC_OK;
       });
     });
@@ -895,7 +901,7 @@ int fc_jpeg_view(const void* store, int store_dtype, const float* scales, int64_
                  void* stream) {
   if (n_tail < 0 || n_tail >= r || (n_tail && !tail)) return FC_ERR_ARG;
   TailRows rows;
-  if (n_tail) rows = TailRows{tail, H * r * D, r * D, D, -1, (int)n_tail};
+  if (n_tail) rows = TailRows{tail, H * r * D, r * D, (int)n_tail};
   const int64_t T = nblk * r + n_tail;
   return jpeg_decode_launch(store, store_dtype, scales, B, H, cap, 0, nblk, D, r, k, basis, out,
                             out_dtype, H * T * D, T * D, D, nblk * r, stream, group, rows);

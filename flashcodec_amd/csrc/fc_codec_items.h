@@ -26,26 +26,14 @@ __device__ __forceinline__ ItemMap item_of_thread(int lpi_log2) {
   return m;
 }
 
-// Raw-tail rows a reconstruction appends to its output (fc_jpeg_view): item
-// `at` of every sequence (one past its archived blocks; -1: none) copies the
-// n tail tokens behind them.
+// Raw-tail rows a reconstruction appends to its output (fc_jpeg_view): the
+// item after the archived blocks of every sequence copies the n contiguous
+// tail tokens behind them.
 struct TailRows {
   const void* p = nullptr;
-  int64_t sb = 0, sh = 0, st = 0;  // elements
-  int64_t at = -1;
+  int64_t sb = 0, sh = 0;  // elements
   int n = 0;
 };
-
-// copies the tail rows of sequence (b, h), VEC features at d0; dst is the
-// sequence's output row 0 at d0
-template <typename TO, int VEC>
-__device__ __forceinline__ void copy_tail(const TailRows& tail, int64_t b, int64_t h, int64_t d0,
-                                          TO* dst, int64_t tok0, int64_t oss) {
-  const TO* src = static_cast<const TO*>(tail.p) + b * tail.sb + h * tail.sh + d0;
-  for (int t = 0; t < tail.n; ++t)
-    *reinterpret_cast<vec_t<TO, VEC>*>(dst + (tok0 + t) * oss) =
-        *reinterpret_cast<const vec_t<TO, VEC>*>(src + t * tail.st);
-}
 
 // Quantizer of an archive: none (coefficients in the stream dtype), one
 // scale per row, one scale per 32 features.
@@ -70,31 +58,40 @@ __device__ __forceinline__ vec_t<T, VEC> round_row(const float (&v)[VEC]) {
   return o;
 }
 
+// Kernel arguments besides the arrays: kept small, since a call of a few
+// microseconds waits for them (see fc_jpeg_decode.hip).
+struct JpegEncodeArgs {
+  int64_t sb, sh, ss, H, m, D, s_valid, cap, n0, items;
+  int k, lpi_log2;
+};
+
 struct JpegEncodeLaunch {
+  JpegEncodeArgs p;
   const void* x;
-  int dtype;
-  int64_t sb, sh, ss, H, m, D, s_valid;
-  int r, k;
+  int dtype, r;
   const float* basis;
   void* out;
   float* scales;
-  int64_t cap, n0, items;
-  int lpi_log2, vec;
+  int vec;
   JpegMode mode;
   const int64_t* gate;  // device (n_blocks, n_tail) of a gated decode-step archive, or NULL
   hipStream_t stream;
 };
 
+struct JpegDecodeArgs {
+  int64_t H, cap, a, nper, D;  // nper: items per sequence (blocks, and the tail's)
+  int64_t osb, osh, oss, out_len, items;
+  int r, k, lpi_log2;
+};
+
 struct JpegDecodeLaunch {
+  JpegDecodeArgs p;
   const void* store;
   int in_dtype, out_dtype;
   const float* scales;
-  int64_t H, cap, a, nper, D;  // nper: items per sequence (blocks, and the tail's)
-  int r, k;
   const float* basis;
   void* out;
-  int64_t osb, osh, oss, out_len, items;
-  int lpi_log2, vec;
+  int vec;
   JpegMode mode;
   TailRows tail;
   hipStream_t stream;
@@ -107,7 +104,7 @@ int jpeg_vec_fast(int dtype, int vec, int64_t D);
 bool jpeg_encode_fast_supported(int r, int dtype, int vec, JpegMode mode, bool whole,
                                 bool gated);
 int jpeg_encode_fast(const JpegEncodeLaunch& a);
-bool jpeg_decode_fast_supported(int k, int out_dtype, int vec, JpegMode mode);
+bool jpeg_decode_fast_supported(int r, int k, int out_dtype, int vec, JpegMode mode);
 int jpeg_decode_fast(const JpegDecodeLaunch& a);
 
 }  // namespace fc

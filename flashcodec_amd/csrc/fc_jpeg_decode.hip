@@ -5,11 +5,16 @@
 // coefficient rows and scales of a block are all requested before the first
 // is used, the tokens formed 8 at a time (64 or 32 accumulators, so blocks of
 // any size fit the registers), rows written with nontemporal stores.
-// 67 MB of bf16 tokens (4 x 8 x 8192 x 128), general kernel -> this one: int8
-// per row k = 4 of 16 24.0 -> 16.2 us, k = 2 of 4 23.3 -> 17.5 us, per 32
-// features k = 4 of 8 23.9 -> 17.7 us, k = 8 of 32 61.7 -> 24.4 us;
-// coefficients k = 4 of 8 24.0 -> 19.2 us, k = 4 of 16 24.6 -> 17.4 us; fp32
-// tokens from int8, k = 4 of 8 59.9 -> 28.3 us (4 elements a lane, not 8).
+// Small calls wait for the kernel's arguments and its first loads: the
+// arguments are few, and the tail rows of a view are a variant of their own
+// (with both at run time calls of 3-5 us took 3% longer).  Stored rows are
+// unrolled, except above 4 in blocks of 16 or of other sizes: guards on a
+// runtime count held k = 8 of 8 bf16 coefficients at 18.5 us for 34 MB of
+// tokens, 13.4 now, the general kernel 17.3 (in the caches 14.2, 9.4, 14.6).
+// 34 MB of bf16 tokens (32 x 4096 x 128), general kernel -> this one, archive
+// not in the caches: coefficients k = 2 of 8 11.4 -> 8.2 us, k = 4 13.7 -> 9.5,
+// k = 4 of 16 14.2 -> 10.0; int8 per row k = 4 of 16 16.9 -> 11.7, per 32
+// features k = 4 of 8 16.3 -> 12.1.
 #include "fc_codec_items.h"
 
 namespace fc {
@@ -18,6 +23,8 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+struct NoTail {};
 
 template <int BYTES>
 struct nt_word {
@@ -40,29 +47,14 @@ __device__ __forceinline__ void nt_store_row(TO* p, const float (&v)[VEC]) {
   }
 }
 
-// VEC stored elements of a row, read once
-template <typename TI, int VEC>
-__device__ __forceinline__ vec_t<TI, VEC> nt_load_row(const TI* p) {
-  if constexpr (sizeof(vec_t<TI, VEC>) == 32) {
-    struct Two { u32x4 a, b; };
-    return __builtin_bit_cast(
-        vec_t<TI, VEC>,
-        Two{__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)),
-            __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p) + 1)});
-  } else {
-    typedef typename nt_word<sizeof(vec_t<TI, VEC>)>::type W;
-    return __builtin_bit_cast(vec_t<TI, VEC>,
-                              __builtin_nontemporal_load(reinterpret_cast<const W*>(p)));
-  }
-}
-
 // R: tokens per block, 0 = runtime r (tokens formed 8 at a time); KT: kept
 // frequencies, 0 = runtime k <= 8.  The arrays come as restrict arguments
 // besides the launch description (loads ahead of the stores).
-template <typename TI, typename TO, int VEC, int R, int KT, bool GROUP>
+template <typename TI, typename TO, int VEC, int R, int KT, bool GROUP, bool TAIL>
 __global__ __launch_bounds__(kThreads) void jpeg_decode_fast_kernel(
     const TI* __restrict__ store, const float* __restrict__ scales,
-    const float* __restrict__ basis, TO* __restrict__ out, JpegDecodeLaunch p) {
+    const float* __restrict__ basis, TO* __restrict__ out, JpegDecodeArgs p,
+    std::conditional_t<TAIL, TailRows, NoTail> tail) {
   constexpr bool QUANT = std::is_same<TI, int8_t>::value;
   constexpr int KMAX = KT > 0 ? KT : 8;
   constexpr int TB = R > 0 && R < 8 ? R : 8;  // tokens formed at a time
@@ -76,16 +68,27 @@ __global__ __launch_bounds__(kThreads) void jpeg_decode_fast_kernel(
   if (d0 >= p.D) return;
   TO* const seq = out + b * p.osb + h * p.osh + d0;
   const int64_t tok0 = blk * r;
-  if (rel == p.tail.at) return copy_tail<TO, VEC>(p.tail, b, h, d0, seq, tok0, p.oss);
+  if constexpr (TAIL) {
+    if (rel + 1 == p.nper) {
+      const TO* src = static_cast<const TO*>(tail.p) + b * tail.sb + h * tail.sh + d0;
+      for (int t = 0; t < tail.n; ++t)
+        *reinterpret_cast<vec_t<TO, VEC>*>(seq + (tok0 + t) * p.oss) =
+            *reinterpret_cast<const vec_t<TO, VEC>*>(src + t * p.D);
+      return;
+    }
+  }
   const int64_t row0 = (bh * p.cap + blk) * k;
   const TI* src = store + row0 * p.D + d0;
 
-  vec_t<TI, VEC> q[KMAX];
+  // rows are read past the caches: 2-9% faster than with ordinary loads, more
+  // for many codes (67 MB of bf16 tokens, int8 k = 8 of 8, 23.8 us for 28.6)
+  typedef typename nt_word<sizeof(vec_t<TI, VEC>)>::type W;
+  W q[KMAX];
   float s[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j < k) {
-      q[j] = nt_load_row<TI, VEC>(src + (int64_t)j * p.D);
+      q[j] = __builtin_nontemporal_load(reinterpret_cast<const W*>(src + (int64_t)j * p.D));
       if constexpr (QUANT)
         s[j] = GROUP ? scales[(row0 + j) * (p.D / 32) + d0 / 32] : scales[row0 + j];
     }
@@ -102,9 +105,20 @@ __global__ __launch_bounds__(kThreads) void jpeg_decode_fast_kernel(
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) {
       if (j < k) {
+        // (more than 4 rows: the conversion stays with its tokens, hoisted past
+        // them it takes 64 registers)
+        if constexpr (KMAX > 4 && R != 8) {
+#pragma unroll
+          for (int i = 0; i < (int)(sizeof(W) / 4); ++i) {
+            uint32_t x = q[j][i];
+            asm("" : "+v"(x));
+            q[j][i] = x;
+          }
+        }
+        const vec_t<TI, VEC> row = __builtin_bit_cast(vec_t<TI, VEC>, q[j]);
         float c[VEC];
 #pragma unroll
-        for (int v = 0; v < VEC; ++v) c[v] = QUANT ? to_f32(q[j].v[v]) * s[j] : to_f32(q[j].v[v]);
+        for (int v = 0; v < VEC; ++v) c[v] = QUANT ? to_f32(row.v[v]) * s[j] : to_f32(row.v[v]);
         const float* mj = basis + j * r + t0;
 #pragma unroll
         for (int t = 0; t < TB; ++t) {
@@ -125,28 +139,49 @@ __global__ __launch_bounds__(kThreads) void jpeg_decode_fast_kernel(
 
 template <typename TI, typename TO, int VEC, bool GROUP>
 void launch(const JpegDecodeLaunch& a) {
-  const int64_t per = kThreads >> a.lpi_log2;
-  const dim3 grid((unsigned)((a.items + per - 1) / per));
+  const int64_t per = kThreads >> a.p.lpi_log2;
+  const dim3 grid((unsigned)((a.p.items + per - 1) / per));
+  auto go = [&](auto rc, auto kc) {
+    constexpr int R = decltype(rc)::value, KT = decltype(kc)::value;
+    const TI* store = static_cast<const TI*>(a.store);
+    TO* out = static_cast<TO*>(a.out);
+    // (a view is in the stream dtype: int8 codes, or rows of the same type)
+    if constexpr (std::is_same<TI, int8_t>::value || std::is_same<TI, TO>::value) {
+      if (a.tail.n) {
+        jpeg_decode_fast_kernel<TI, TO, VEC, R, KT, GROUP, true>
+            <<<grid, kThreads, 0, a.stream>>>(store, a.scales, a.basis, out, a.p, a.tail);
+        return;
+      }
+    }
+    jpeg_decode_fast_kernel<TI, TO, VEC, R, KT, GROUP, false>
+        <<<grid, kThreads, 0, a.stream>>>(store, a.scales, a.basis, out, a.p, NoTail{});
+  };
+  using std::integral_constant;
   auto with_k = [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    if (a.k == 2)
-      jpeg_decode_fast_kernel<TI, TO, VEC, R, 2, GROUP><<<grid, kThreads, 0, a.stream>>>(
-          static_cast<const TI*>(a.store), a.scales, a.basis, static_cast<TO*>(a.out), a);
-    else if (a.k == 4)
-      jpeg_decode_fast_kernel<TI, TO, VEC, R, 4, GROUP><<<grid, kThreads, 0, a.stream>>>(
-          static_cast<const TI*>(a.store), a.scales, a.basis, static_cast<TO*>(a.out), a);
-    else if (R == 8 && std::is_same<TI, int8_t>::value && !GROUP && a.k == 8)
-      jpeg_decode_fast_kernel<int8_t, TO, VEC, 8, 8, false><<<grid, kThreads, 0, a.stream>>>(
-          static_cast<const int8_t*>(a.store), a.scales, a.basis, static_cast<TO*>(a.out), a);
-    else
-      jpeg_decode_fast_kernel<TI, TO, VEC, R, 0, GROUP><<<grid, kThreads, 0, a.stream>>>(
-          static_cast<const TI*>(a.store), a.scales, a.basis, static_cast<TO*>(a.out), a);
+    switch (a.p.k) {
+      case 1: return go(rc, integral_constant<int, 1>{});
+      case 2: return go(rc, integral_constant<int, 2>{});
+      case 3: return go(rc, integral_constant<int, 3>{});
+      case 4: return go(rc, integral_constant<int, 4>{});
+      default: break;
+    }
+    if constexpr (R == 8) {
+      switch (a.p.k) {
+        case 5: return go(rc, integral_constant<int, 5>{});
+        case 6: return go(rc, integral_constant<int, 6>{});
+        case 7: return go(rc, integral_constant<int, 7>{});
+        default: return go(rc, integral_constant<int, 8>{});
+      }
+    } else if constexpr (R != 4) {
+      go(rc, integral_constant<int, 0>{});
+    }
   };
-  switch (a.r) {
-    case 4: with_k(std::integral_constant<int, 4>{}); break;
-    case 8: with_k(std::integral_constant<int, 8>{}); break;
-    case 16: with_k(std::integral_constant<int, 16>{}); break;
-    default: with_k(std::integral_constant<int, 0>{}); break;
+  switch (a.p.r) {
+    case 4: with_k(integral_constant<int, 4>{}); break;
+    case 8: with_k(integral_constant<int, 8>{}); break;
+    case 16: with_k(integral_constant<int, 16>{}); break;
+    default: with_k(integral_constant<int, 0>{}); break;
   }
 }
 
@@ -154,36 +189,33 @@ template <typename TO, int VEC>
 int launch_out(const JpegDecodeLaunch& a) {
   if constexpr (sizeof(TO) * VEC == 32) {  // fp32 rows of more than 64 lanes x 4
     launch<int8_t, TO, VEC, false>(a);
-    return FC_OK;
-  }
-  if (a.mode == kJpegRow) {
+  } else if (a.mode == kJpegRow) {
     launch<int8_t, TO, VEC, false>(a);
-    return FC_OK;
-  }
-  if (a.mode == kJpegGroup) {
+  } else if (a.mode == kJpegGroup) {
     launch<int8_t, TO, VEC, true>(a);
-    return FC_OK;
-  }
-  if (a.in_dtype == a.out_dtype) {
+  } else if (a.in_dtype == a.out_dtype) {
     launch<TO, TO, VEC, false>(a);
-    return FC_OK;
-  }
-  if constexpr (std::is_same<TO, float>::value) {  // 16-bit coefficients to fp32 tokens
+  } else if constexpr (std::is_same<TO, float>::value) {  // 16-bit coefficients to fp32 tokens
     if (a.in_dtype == FC_F16)
       launch<f16_t, float, VEC, false>(a);
     else
       launch<bf16_t, float, VEC, false>(a);
-    return FC_OK;
   } else {
     return FC_ERR_UNSUPPORTED;
   }
+  return FC_OK;
 }
 
 }  // namespace
 
-bool jpeg_decode_fast_supported(int k, int out_dtype, int vec, JpegMode mode) {
-  if (out_dtype == FC_F32 && vec == 8) return k <= 8 && mode == kJpegRow;
-  return k <= 8 && vec == (out_dtype == FC_F32 ? 4 : 8);
+// fp32 tokens of 16-token blocks with 1 stored row keep the general kernel
+// and its plain stores: 67 MB of tokens at D = 256 take 23.5 us there, 26.5
+// here, 2 MB 4.1 both (k = 2: 24.2 and 25, 2 MB 5.0 and 3.7).
+bool jpeg_decode_fast_supported(int r, int k, int out_dtype, int vec, JpegMode mode) {
+  if (k > 8) return false;
+  if (out_dtype != FC_F32) return vec == 8;
+  if (vec == 8) return mode == kJpegRow;  // rows of more than 64 lanes x 4
+  return vec == 4 && !(r == 16 && k == 1);
 }
 
 int jpeg_decode_fast(const JpegDecodeLaunch& a) {

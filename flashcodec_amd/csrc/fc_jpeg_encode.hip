@@ -140,12 +140,12 @@ __device__ __forceinline__ void nt_store_row(T* p, const float (&v)[VEC]) {
 template <typename T, int VEC, int R, int KT, JpegMode MODE, bool GATED>
 __global__ __launch_bounds__(kThreads) void jpeg_encode_fast_kernel(
     const T* __restrict__ x, const float* __restrict__ basis, void* __restrict__ out,
-    float* __restrict__ scales, JpegEncodeLaunch p) {
+    float* __restrict__ scales, JpegEncodeArgs p, const int64_t* __restrict__ gate) {
   int64_t n0 = p.n0;
   if constexpr (GATED) {
     // gate = device (n_blocks, n_tail): archive only a completed tail
-    if (p.gate[1] != R - 1) return;
-    n0 = p.gate[0];
+    if (gate[1] != R - 1) return;
+    n0 = gate[0];
     if (n0 < 0 || n0 + p.m > p.cap) return;
   }
   const int k = KT > 0 ? KT : p.k;
@@ -228,20 +228,20 @@ __global__ __launch_bounds__(kThreads) void jpeg_encode_fast_kernel(
 
 template <typename T, int VEC, int R, JpegMode MODE, bool GATED>
 void launch(const JpegEncodeLaunch& a) {
-  const int64_t per = kThreads >> a.lpi_log2;
-  const dim3 grid((unsigned)((a.items + per - 1) / per));
-  if (a.k == 2)
+  const int64_t per = kThreads >> a.p.lpi_log2;
+  const dim3 grid((unsigned)((a.p.items + per - 1) / per));
+  if (a.p.k == 2)
     jpeg_encode_fast_kernel<T, VEC, R, 2, MODE, GATED><<<grid, kThreads, 0, a.stream>>>(
-        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a);
-  else if (a.k == 4)
+        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a.p, a.gate);
+  else if (a.p.k == 4)
     jpeg_encode_fast_kernel<T, VEC, R, 4, MODE, GATED><<<grid, kThreads, 0, a.stream>>>(
-        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a);
-  else if (R == 8 && MODE == kJpegRow && a.k == 8)
+        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a.p, a.gate);
+  else if (R == 8 && MODE == kJpegRow && a.p.k == 8)
     jpeg_encode_fast_kernel<T, VEC, 8, 8, kJpegRow, GATED><<<grid, kThreads, 0, a.stream>>>(
-        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a);
+        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a.p, a.gate);
   else
     jpeg_encode_fast_kernel<T, VEC, R, 0, MODE, GATED><<<grid, kThreads, 0, a.stream>>>(
-        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a);
+        static_cast<const T*>(a.x), a.basis, a.out, a.scales, a.p, a.gate);
 }
 
 template <typename T, int VEC>

@@ -127,7 +127,8 @@ int fc_jpeg_decode_grouped(const int8_t* codes, const float* scales,
                            int64_t out_len, void* stream);
 
 /*
- * The whole view of a stream with a raw tail in one launch: blocks
+ * The whole view of a stream with a raw tail (one launch where the
+ * register-resident read kernel takes the shape, else two): blocks
  * [0, nblk) reconstructed into the contiguous out (B, H, nblk*r + n_tail, D)
  * (as fc_jpeg_decode; group 32: per-group scales, 0: one per row), then the
  * first n_tail < r rows of the contiguous tail buffer (B, H, r, D)

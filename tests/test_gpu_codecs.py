@@ -439,13 +439,18 @@ def test_quantizer_nan_and_inf(dt, oracle):
 FAST_EDGES = [
     # dtype, r, k, D, S, group: the register-resident kernels' block sizes
     # and kept-frequency variants, rows that leave lanes idle, a ragged last
-    # block; k = 9 and D = 12 in 16 bits leave them for the general kernels
+    # block; k = 9, D = 12 in 16 bits and (to fp32 tokens) 1 row of 16-token
+    # blocks leave them for the general kernels
     ("bf16", 4, 1, 8, 4 * 65 + 3, 0), ("f16", 4, 2, 80, 4 * 33 + 1, 0),
     ("f32", 4, 4, 128, 4 * 40, 32), ("bf16", 8, 3, 96, 8 * 31 + 5, 32),
     ("f16", 8, 8, 256, 8 * 9 + 7, 0), ("f32", 8, 2, 20, 8 * 70 + 1, 0),
     ("f32", 8, 4, 512, 8 * 5 + 2, 0), ("f32", 8, 5, 256, 8 * 6, 32),
     ("bf16", 16, 4, 128, 16 * 20 + 15, 0), ("f32", 16, 2, 64, 16 * 17 + 1, 32),
     ("f16", 16, 9, 64, 16 * 7 + 3, 0), ("bf16", 8, 4, 12, 8 * 9 + 4, 0),
+    ("bf16", 8, 1, 64, 8 * 21 + 1, 32), ("f16", 8, 6, 128, 8 * 12 + 2, 32),
+    ("bf16", 8, 7, 40, 8 * 15 + 3, 0), ("bf16", 16, 1, 128, 16 * 9 + 5, 0),
+    ("f32", 16, 2, 256, 16 * 4 + 6, 0), ("f32", 16, 3, 64, 16 * 6 + 2, 0),
+    ("f16", 4, 3, 128, 4 * 21 + 1, 32), ("f32", 6, 1, 64, 6 * 13 + 5, 0),
     ("f16", 32, 8, 128, 32 * 3 + 9, 0), ("f32", 5, 2, 128, 5 * 11 + 2, 0),
 ]
 
