@@ -347,20 +347,17 @@ class _CodecStream:
         return view if not self._n_raw else torch.cat([view, self.raw], dim=-2)
 
     def _joined_view(self, tail):
-        """A fresh view of archive + raw tail in one launch.  A jpeg archive
-        of at most half the tokens' bytes (and the block sizes of the
-        register-resident kernels) is reconstructed straight into it, the
-        others copy _rec: for 67 MB of 16-bit tokens the copy takes 21.1 us,
-        the reconstruction 16.8 us (int8, k = 4 of 8), 20.6 us (int8, k = 8),
-        19.2 us (bf16 coefficients, k = 4) and 30.0 us (k = 8)."""
+        """A fresh view of archive + raw tail: reconstructed into it from the
+        archive in one launch where that is the faster route (_reads_archive),
+        else _rec and the tail copied into it."""
         c, t = self.codec, self._n_raw
-        r, k = c.block_size, getattr(c, "keep_freqs", 0)
+        r = c.block_size
         B, H, _, D = tail.shape
         es, L = tail.element_size(), N.lib()
         out = tail.new_empty((B, H, self.n_archived + t, D))
         stream = N.stream_ptr(tail.device)
-        if k and k <= 8 and r in (4, 8, 16) and (2 * k * (1 if c.quantized else es) <= r * es):
-            code = N.dtype_code(tail.dtype)
+        if self._reads_archive(D, es, out.numel() * es):
+            k, code = c.keep_freqs, N.dtype_code(tail.dtype)
             rc = L.fc_jpeg_view(
                 self._coeffs.data_ptr(), N.I8 if c.quantized else code, N.ptr(self._scales), B, H,
                 self._capacity, self.n_blocks, D, r, k, c.quant_group,
@@ -375,6 +372,22 @@ class _CodecStream:
                               B * H, stream)
         N.check(rc, "fc_concat_rows")
         return out
+
+    def _reads_archive(self, D, es, nbytes):
+        """Whether a joined view of `nbytes` is faster reconstructed than
+        copied from _rec.  Both read less than they write; the copy starts
+        sooner and has no arithmetic, so it wins until its extra reads cost
+        more: bf16, k = 4 of 8 int8, 2 MB 2.8 us against 4.0, 17 MB 4.7 : 6.0
+        (7.8 : 7.3 with nothing in the caches), 34 MB 9.3 : 8.2 (13.8 : 10.7),
+        67 MB 20.3 : 12.9, 134 MB 39.3 : 26.7.  Reconstructed: from 32 MiB,
+        archives of at most half the tokens' bytes whose kernel has all stored
+        rows unrolled (k = 8 of 16: 67 MB 23.0 us, the copy 20.3) and rows that
+        fill its 16-byte lanes (D = 100 in bf16, 26 MB: 13.8 us, the copy 8.8)."""
+        c = self.codec
+        r, k = c.block_size, getattr(c, "keep_freqs", 0)
+        return (nbytes >= 1 << 25 and 0 < k and (k <= 4 or r == 8) and r in (4, 8, 16)
+                and 2 * k * (1 if c.quantized else es) <= r * es
+                and (D % 8 == 0 if es == 2 else D % 4 == 0 and D <= 256))
 
     # ------------------------------------------------------------ structure
     def reset(self):

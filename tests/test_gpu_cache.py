@@ -10,7 +10,9 @@ import pytest
 import torch
 
 import flashcodec_amd as fc
+from flashcodec_amd import _native as N
 from flashcodec_amd.cache import _CodecStream
+from flashcodec_amd.codecs import jpeg as jp
 from tests.conftest import Golden, bits, to_torch, to_values
 
 pytestmark = pytest.mark.gpu
@@ -271,14 +273,17 @@ def test_tail_reads_are_copies_and_follow_batch_changes(seqs):
 
 
 VIEW_CASES = [
-    # (codec options, dtype, D, blocks, tail): the joined view reconstructs
-    # from the archive (int8, or fewer coefficients than tokens) or copies
-    # the reconstruction; 16-, 4- and 1-byte words of the copy
+    # (codec options, dtype, D, blocks, tail): the copy of the reconstruction
+    # and the tail in 16-, 4- and 1-byte words; the jpeg ones also through
+    # fc_jpeg_view, by its register-resident and its general kernel
     (dict(mode="jpeg", block_size=8, keep_freqs=4, quant_bits=8), torch.float16, 128, 37, 7),
     (dict(mode="jpeg", block_size=8, keep_freqs=3, quant_bits=8), torch.bfloat16, 80, 5, 1),
     (dict(mode="jpeg", block_size=16, keep_freqs=4, quant_bits=8, quant_group=32), torch.bfloat16,
      96, 9, 15),
     (dict(mode="jpeg", block_size=8, keep_freqs=2), torch.float32, 64, 33, 3),
+    (dict(mode="jpeg", block_size=8, keep_freqs=5, quant_bits=8), torch.float16, 256, 17, 2),
+    (dict(mode="jpeg", block_size=16, keep_freqs=1), torch.float32, 128, 6, 9),
+    (dict(mode="jpeg", block_size=8, keep_freqs=4, quant_bits=8), torch.bfloat16, 12, 9, 6),
     (dict(mode="jpeg", block_size=4, keep_freqs=4), torch.bfloat16, 128, 130, 2),
     (dict(mode="jpeg", block_size=8, keep_freqs=8), torch.float16, 6, 3, 5),
     (dict(mode="jpeg", block_size=5, keep_freqs=5), torch.bfloat16, 7, 11, 4),
@@ -302,8 +307,43 @@ def test_view_with_tail_is_reconstruction_then_tail(cfg, dt, D, nb, tail):
     want = torch.cat([rec, x[:, :, nb * r:]], dim=-2)
     got = st.read()
     assert got.is_contiguous() and torch.equal(got, want)
+    if cfg["mode"] == "jpeg":
+        one = torch.full_like(want, float("nan"))
+        k, code = cfg["keep_freqs"], N.dtype_code(dt)
+        rc = N.lib().fc_jpeg_view(
+            st._coeffs.data_ptr(), N.dtype_code(st._coeffs.dtype), N.ptr(st._scales), B, H,
+            st._capacity, nb, D, r, k, st.codec.quant_group, jp.device_basis(r, k, DEV).data_ptr(),
+            st._raw_buf.data_ptr(), tail, one.data_ptr(), code, N.stream_ptr(one.device))
+        assert rc == N.OK and torch.equal(one, want)
     st.append(x[:, :, :r])                      # completes the block, new tail
     assert torch.equal(got, want)
     again = st.read()
     assert torch.equal(again[:, :, :nb * r], rec)
     assert torch.equal(again[:, :, (nb + 1) * r:], x[:, :, r - tail:r])
+
+
+ROUTE_I8 = dict(mode="jpeg", block_size=8, keep_freqs=4, quant_bits=8)
+
+
+@pytest.mark.parametrize("cfg,dt,D,H,nb,from_archive", [
+    (ROUTE_I8, torch.bfloat16, 128, 8, 64, False),                    # 1 MB
+    (ROUTE_I8, torch.bfloat16, 128, 32, 511, False),                  # 5 rows a head under 32 MiB
+    (ROUTE_I8, torch.bfloat16, 128, 32, 512, True),
+    (ROUTE_I8, torch.bfloat16, 100, 32, 700, False),                  # rows of no whole 16-byte lanes
+    (dict(ROUTE_I8, quant_bits=0), torch.float32, 256, 16, 257, True),
+    (dict(ROUTE_I8, block_size=16, keep_freqs=8, quant_bits=0), torch.bfloat16, 128, 32, 260, False),
+])
+def test_joined_view_route(cfg, dt, D, H, nb, from_archive):
+    """Views from 32 MiB are reconstructed from the archive, the others (whose
+    copy is the faster one) copied from the memoised reconstruction; both bit
+    for bit reconstruction and tail."""
+    r, tail = cfg["block_size"], 3
+    g = torch.Generator(device=DEV).manual_seed(nb)
+    x = torch.randn((1, H, nb * r + tail, D), generator=g, device=DEV).to(dt)
+    st = _CodecStream(fc.make_codec(**cfg))
+    st.append(x)
+    got = st.read()
+    assert (st._rec is None) == from_archive
+    rec = torch.empty((1, H, nb * r, D), dtype=dt, device=DEV)
+    st._reconstruct(0, nb, rec, nb * r)
+    assert torch.equal(got, torch.cat([rec, x[:, :, nb * r:]], dim=-2))
