@@ -58,6 +58,7 @@ def sources():
 FILE_FLAGS = {
     "fc_attn_mfma": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "fc_prefill": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    **{f"fc_attn_fpj_d{d}.": ["-mllvm", "-amdgpu-mfma-vgpr-form"] for d in (80, 96, 256)},
 }
 
 

@@ -18,7 +18,7 @@ from flashcodec_amd import _native as N
 from flashcodec_amd import attention as fa
 from flashcodec_amd.cache import _CodecStream
 from tests.conftest import to_values, torch_dtype
-from tests.test_gpu_attention import assert_close, build_streams, oracle_out
+from tests.test_gpu_attention import HALF_ULP, assert_close, build_streams, oracle_out
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -517,8 +517,9 @@ def test_c5_full_shape_materialization_free_tracks_materialized():
 FPJ_WIDTHS = [
     # dtype, r, k, G, D, tokens: the fp-coefficient pass's head sizes besides
     # 64 / 128; less than a pass, ragged passes, k = 3 (whole blocks only), one
-    # and two groups of query heads, a raw tail or none
+    # and two groups of query heads, 16 heads at D = 256, a raw tail or none
     ("bf16", 8, 2, 4, 256, 8 * 1500 + 5), ("f16", 8, 4, 8, 256, 8 * 700), ("bf16", 4, 1, 1, 256, 4 * 9 + 3),
+    ("bf16", 8, 8, 16, 256, 8 * 150 + 3), ("f16", 16, 4, 12, 256, 16 * 61 + 9),
     ("f16", 8, 3, 3, 256, 8 * 333 + 1), ("f16", 8, 8, 2, 80, 8 * 260 + 7), ("bf16", 16, 2, 20, 80, 16 * 90 + 15),
     ("bf16", 8, 3, 6, 96, 8 * 411 + 2), ("f16", 4, 4, 16, 96, 4 * 1200), ("f16", 16, 1, 2, 96, 16 * 3 + 1),
 ]
@@ -554,3 +555,27 @@ def test_fp_coefficient_widths_on_matrix_cores(dt, r, k, G, D, S, oracle, attent
         _archives_equal(ks, kr)
         _archives_equal(vs, vr)
         assert_close(to_values(o)[:, :, 0], oracle_out(oracle, qt, ks, vs, D ** -0.5), dt)
+
+
+@pytest.mark.parametrize("D", [80, 96, 256])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+def test_fp_coefficient_widths_small_weights(dt, D, oracle):
+    """3200 tokens of weight e^-14 and one block of zero values that holds all
+    the rest of the softmax: the sum over the small weights is the output, so
+    their relative error is its.  Within an ulp of the output (half for its
+    rounding, the rest for fp32 exponentials and sums)."""
+    B, Hkv, G, r, n = 1, 2, 4, 8, 401
+    print(f"case fp widths small weights {dt} D={D}", flush=True)
+    codec = fc.make_codec(mode="jpeg", block_size=r, keep_freqs=1)
+    g = torch.Generator(device=DEV).manual_seed(47 + D)
+    kx = torch.zeros((B, Hkv, n, r, D), device=DEV)
+    kx[:, :, 0] = 14.0 * D ** -0.5
+    vx = 512 * (1 + torch.rand((B, Hkv, n, 1, D), generator=g, device=DEV)).expand(B, Hkv, n, r, D).clone()
+    vx[:, :, 0] = 0
+    ks, vs = _CodecStream(codec), _CodecStream(codec)
+    for st, x in ((ks, kx), (vs, vx)):
+        st.append(x.reshape(B, Hkv, n * r, D).to(torch_dtype(dt)))
+    q = torch.ones((B, Hkv * G, 1, D), device=DEV, dtype=torch_dtype(dt))
+    out = to_values(fc.codec_decode_attention(q, ks, vs))[:, :, 0]
+    ref = oracle_out(oracle, q, ks, vs, D ** -0.5)
+    assert (np.abs(out - ref) <= 2 * HALF_ULP[dt] * np.abs(ref)).all(), (np.abs(out / ref - 1)).max()
