@@ -501,7 +501,7 @@ __device__ __forceinline__ void fused_merge(const MfmaArgs& p, int64_t b, int64_
     float pmv[kPre], plv[kPre];
 #pragma unroll
     for (int j = 0; j < kPre; ++j) {
-      const int sp = j < ns ? j : 0;
+      const int sp = j < ns ? j : G * ns;  // none such: zero (another's may be infinite)
       pa[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
                                                rp, ((h * ns + sp) * C4 + c) * 16, 0, kCachePolicySc1));
       pmv[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (h * ns + sp) * 4, 0,
@@ -586,7 +586,7 @@ __device__ __forceinline__ void wide_merge(const MfmaArgs& p, int64_t b, int64_t
   float4_t pa[NH];
 #pragma unroll
   for (int j = 0; j < NH; ++j) {
-    const int sp = s0 + j < ns ? s0 + j : 0;
+    const int sp = s0 + j < ns ? s0 + j : G * ns;  // none such: zero
     pa[j] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
                                              rp, ((h * ns + sp) * C4 + c) * 16, 0, kCachePolicySc1));
   }

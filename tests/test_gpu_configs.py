@@ -579,3 +579,22 @@ def test_fp_coefficient_widths_small_weights(dt, D, oracle):
     out = to_values(fc.codec_decode_attention(q, ks, vs))[:, :, 0]
     ref = oracle_out(oracle, q, ks, vs, D ** -0.5)
     assert (np.abs(out - ref) <= 2 * HALF_ULP[dt] * np.abs(ref)).all(), (np.abs(out / ref - 1)).max()
+
+
+@pytest.mark.parametrize("D,k", [(80, 2), (96, 1), (256, 4)])
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+def test_fp_coefficient_widths_infinite_values(dt, D, k, oracle, attention_pass):
+    """An infinite value coefficient gives the infinities (by the sign of its
+    weight) and nothing else the vector-ALU pass gives."""
+    B, Hkv, G, r = 2, 2, 4, 8
+    print(f"case fp widths infinities {dt} D={D} k={k}", flush=True)
+    cfg = dict(mode="jpeg", block_size=r, keep_freqs=k)
+    ks, vs = build_streams(cfg, dt, B, Hkv, r * 300 + 3, D, 53 + D, oracle)
+    vs._coeffs[:, :, 5, 0, 3] = float("inf")
+    vs._coeffs[:, :, 290, k - 1, D - 1] = float("-inf")
+    q = queries(B, Hkv * G, D, 54 + D, dt)
+    out = fc.codec_decode_attention(q, ks, vs).float()
+    attention_pass("valu")
+    ref = fc.codec_decode_attention(q, ks, vs).float()
+    assert int(ref.isinf().sum()) == 2 * B * Hkv * G and not ref.isnan().any()
+    assert torch.equal(out.isinf() * out.sign(), ref.isinf() * ref.sign()) and not out.isnan().any()
