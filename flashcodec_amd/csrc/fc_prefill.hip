@@ -10,11 +10,63 @@ template int launch_prefill<1, 0>(const PrefillArgs&, int, int, int, bool, unsig
 template int launch_prefill<2, 0>(const PrefillArgs&, int, int, int, bool, unsigned, hipStream_t);
 template int launch_prefill<4, 0>(const PrefillArgs&, int, int, int, bool, unsigned, hipStream_t);
 
+// Query heads of a wavefront's 16 queries.
+static int prefill_heads_per_wave(int64_t G) {
+  int gq = 1;
+  while (gq < 16 && G % (2 * gq) == 0) gq *= 2;
+  return gq;
+}
+
+// Compute units of the current device, 0 if it does not say.
+static int device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+    return n;
+  (void)hipGetLastError();
+  return 0;
+}
+
 }  // namespace fc
 
 using namespace fc;
 
 extern "C" {
+
+// The workgroup-shared pass takes D = 64 / 128 and blocks of 4 or 8 tokens (at
+// 16 its 3-wavefront register budget spills and the register-resident pass
+// is faster: 1326 vs 1542 us at 16 x 16 heads x 4096 tokens, D = 128).  With
+// a scale per 32 features at D = 128 it needs two workgroups on some compute
+// units: with one on each it waits at its barriers and LDS round trips (256
+// workgroups, 9192 tokens, 197 us, the register-resident pass 176; 288: 240 and
+// 268; 512: 245 and 270; 1008: 433 and 499).  The grid counts in longest tiles,
+// since its end runs with fewer: a whole prompt of 4096 tokens in 512
+// workgroups (260 of the longest) takes 101 us, in registers 96; 1000 on 300
+// (315) 49.1 and 45.0; 1000 on 1000 (381) 64 and 69.
+// Under 6 passes its longer start counts (485 of 300 tokens 27.6 us, in registers
+// 25.3; 960 of 130 19.3 and 21.0), and wavefronts without tokens load for
+// the others there, which in registers leave (1024 workgroups, 5 of 8 wavefronts
+// with tokens, 1024 tokens: 73.5 and 62.4; 17 of 20, 1280: 62 and 73).
+// D = 64 is as fast or faster shared at every grid (0-58%) but for such short,
+// part-filled ones (512 workgroups, 2 of 4 wavefronts, 130 tokens 15.5 and 14.1).
+int fc_prefill_shared_pass(int store_kind, int r, int s, int64_t D, int64_t B, int64_t Hkv,
+                           int64_t G, int64_t Sq, int64_t P0, int n_cu) {
+  if (B <= 0 || Hkv <= 0 || G <= 0 || Sq <= 0 || P0 < 0) return 0;
+  if (s != 4 || (D != 64 && D != 128) || (r != 4 && r != 8)) return 0;
+  if (store_kind != FC_STORE_JPEG_I8G) return store_kind == FC_STORE_JPEG_I8;
+  if (n_cu <= 0) n_cu = 256;
+  const int64_t gq = prefill_heads_per_wave(G), tq = 16 / gq, tile = 4 * tq;
+  const int64_t nt = (Sq + tile - 1) / tile, cols = G / gq * Hkv * B;
+  const int64_t waves = (Sq + tq - 1) / tq;  // with tokens, of 4 nt
+  const int64_t passes = (P0 + Sq) / (16 * r);
+  if (D == 64) return waves > 2 * nt || passes >= 2 || nt * cols <= n_cu;
+  const bool filled = passes >= 6 ? 5 * waves >= 16 * nt : 3 * waves >= 10 * nt;  // 4/5, 5/6
+  const double work = (double)nt * P0 + 0.5 * tile * nt * (nt - 1) + Sq;  // tokens of all tiles
+  // longest tiles per unit: more where the tiles differ more
+  const double f = (double)Sq / (double)(P0 + Sq);
+  const double need = passes >= 6 ? 1.03125 + 0.375 * f * f : 3.625;
+  return filled && work * cols >= need * n_cu * (double)(P0 + Sq);
+}
 
 int fc_prefill_attention(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_st,
                          int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t D, int64_t P0,
@@ -79,8 +131,7 @@ int fc_prefill_attention(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh,
   a.o_st = o_st;
   // a wavefront's 16 queries: the largest power-of-two head count <= 16
   // that divides G, times 16 / that many consecutive tokens
-  int gq = 1;
-  while (gq < 16 && G % (2 * gq) == 0) gq *= 2;
+  const int gq = prefill_heads_per_wave(G);
   a.gq = gq;
   a.tq = 16 / gq;
   a.hgroups = G / gq;
@@ -91,12 +142,11 @@ int fc_prefill_attention(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh,
   const int dk = (int)(D / 32);
   const unsigned nblocks = (unsigned)blocks;
   int rc;
-  // 4 stored rows per block of 4, 8 or 16 tokens: the softmax on the
-  // matrix cores (one 4x4 product per block); with D = 64 / 128 and blocks
-  // of 4 or 8 tokens the workgroup shares each pass through LDS (at 16
-  // tokens its 3-wavefront register budget spills and the register-resident
-  // pass is faster: 1326 vs 1542 us at 16 x 16 heads x 4096 tokens, D = 128)
-  const bool wg = s == 4 && (D == 64 || D == 128) && (r == 4 || r == 8) && n_raw < r;
+  // 4 stored rows per block of 4, 8 or 16 tokens: the softmax on the matrix
+  // cores (one 4x4 product per block), each pass shared by the workgroup or in
+  // registers
+  const bool wg = n_raw < r && fc_prefill_shared_pass(store_kind, r, s, D, B, Hkv, G, Sq, P0,
+                                                      grouped ? device_cus() : 0) == 1;
   if (wg && r == 8)
     rc = launch_prefill_wg<8>(a, dk, q_dtype, stream_dtype, grouped, nblocks, st);
   else if (wg && r == 4)

@@ -439,6 +439,15 @@ int fc_set_attention_pass(int pass);
 int fc_get_attention_pass(void);
 
 /*
+ * Whether fc_prefill_attention runs a call (fewer than r raw-tail tokens)
+ * with the passes shared by the workgroup (1) or in registers (0) on a device
+ * of n_cu compute units (<= 0: 256); store_kind FC_STORE_JPEG_I8 or _I8G.
+ */
+int fc_prefill_shared_pass(int store_kind, int r, int s, int64_t D, int64_t B,
+                           int64_t Hkv, int64_t G, int64_t Sq, int64_t P0,
+                           int n_cu);
+
+/*
  * Causal prefill attention on int8 jpeg archives without the reconstructed
  * view: the Sq query tokens q (B, Hq, Sq, D) (q_dtype FC_F16 / FC_BF16,
  * element strides q_sb, q_sh, q_st) sit at positions P0 .. P0+Sq-1 of the

@@ -53,6 +53,43 @@ def test_workspace_and_split_policy():
             assert bps * (ns - 1) < nb          # no empty split
 
 
+def test_prefill_pass_rule():
+    """The shared prefill pass with a scale per 32 features at D = 128 needs
+    workgroups mostly filled with tokens and as many longest tiles as compute
+    units and more, the more the tiles differ (29/8 under 6 passes); one scale per row takes it at every
+    grid, D = 64 but for short, part-filled ones."""
+    def shared(kind, D, B, Hkv, G, Sq, P0, r=8, s=4, n_cu=256):
+        return N.lib().fc_prefill_shared_pass(kind, r, s, D, B, Hkv, G, Sq, P0, n_cu)
+    g, row = N.STORE_JPEG_I8G, N.STORE_JPEG_I8
+    assert shared(g, 128, 2, 8, 4, 1000, 8192) == 1
+    assert shared(g, 128, 1, 8, 4, 8, 9184) == 0            # 8 workgroups
+    assert shared(g, 128, 8, 8, 4, 256, 8936) == 1          # 1024 of about the same length
+    assert shared(g, 128, 1, 8, 1, 4096, 0) == 0            # 512, 260 of the longest
+    assert shared(g, 128, 1, 8, 1, 4096, 0, n_cu=128) == 1
+    assert shared(g, 128, 1, 8, 1, 4096, 0, n_cu=0) == 0    # 256 assumed
+    assert shared(g, 128, 64, 8, 4, 20, 1004) == 0          # 5 of 8 wavefronts with tokens
+    assert shared(g, 128, 32, 8, 2, 64, 236) == 0           # 485 of 2 passes
+    assert shared(g, 128, 64, 8, 4, 32, 98) == 1            # 960 of one pass
+    assert shared(g, 64, 64, 8, 4, 8, 122) == 0             # 512, half of their wavefronts
+    assert shared(g, 64, 64, 8, 4, 8, 1000) == 1
+    for B, Hkv, G, Sq, P0 in ((1, 1, 1, 1, 0), (16, 8, 2, 4096, 0), (1, 8, 5, 9, 5000)):
+        assert shared(g, 64, B, Hkv, G, Sq, P0) == 1
+        assert shared(row, 64, B, Hkv, G, Sq, P0, r=4) == 1
+        assert shared(row, 128, B, Hkv, G, Sq, P0) == 1
+        for bad in (dict(r=16), dict(s=2), dict(r=32)):
+            assert shared(row, 128, B, Hkv, G, Sq, P0, **bad) == 0
+        assert shared(row, 256, B, Hkv, G, Sq, P0) == 0
+    for n in (1, 2, 15, 16, 17, 63, 64, 65, 1000):          # against the sum over the tiles
+        for G, cols in ((1, 24), (2, 40), (3, 7), (16, 90)):
+            gq = max(p for p in (1, 2, 4, 8, 16) if G % p == 0)
+            T, P0 = 64 // gq, 2333
+            work = sum(P0 + min(t + T, n) for t in range(0, n, T)) * (G // gq) * cols
+            full = 5 * -(-n // (T // 4)) >= 16 * -(-n // T)
+            f = n / (P0 + n)
+            many = work >= (1.03125 + 0.375 * f * f) * 256 * (P0 + n)
+            assert shared(g, 128, cols, 1, G, n, P0) == (full and many)
+
+
 def test_store_aware_split_count():
     """int8 jpeg stores with half-precision queries take the matrix-core
     split count (at most one round, at least one pass per wavefront, at most

@@ -19,6 +19,7 @@ import pytest
 import torch
 
 import flashcodec_amd as fc
+from flashcodec_amd import _native as N
 from flashcodec_amd.attention import codec_prefill_attention
 from flashcodec_amd.cache import _CodecStream
 from tests.conftest import to_values, torch_dtype
@@ -130,10 +131,11 @@ def test_prefill_matches_causal_attention_on_the_view(case, oracle):
     _prefill_case(case, oracle)
 
 
-# the workgroup-shared pass with a scale per 32 features (4 stored rows, D =
-# 64 / 128, r = 4 / 8).  A pass holds 16 blocks: archives of none, one block, one
-# pass less a block, one pass, a block more, three and four passes and a
-# ragged fifth; 16, 5 (tq = 1) and 1 query heads per kv head
+# 4 stored rows with a scale per 32 features, D = 64 / 128, r = 4 / 8: the
+# workgroup-shared pass on large grids and at D = 64, the register-resident
+# one else.  A pass holds 16 blocks: archives of none, one block, one pass less a
+# block, one pass, a block more, three and four passes and a ragged fifth; 16,
+# 5 (tq = 1) and 1 query heads per kv head
 GROUP_SHARED = [
     ("bf16", 1, 2, 2, 128, 4, 7, 0, 32),
     ("bf16", 1, 1, 4, 128, 4, 8, 0, 32),
@@ -151,6 +153,50 @@ GROUP_SHARED = [
 @pytest.mark.parametrize("case", GROUP_SHARED, ids=[_case_id(c) for c in GROUP_SHARED])
 def test_prefill_group_scales_shared_pass(case, oracle):
     _prefill_case(case, oracle)
+
+
+# grids of workgroups filled with tokens: half a block, one, passes less, of and
+# over 16 blocks, 5 heads (tq = 1), a chunk on a long cache, blocks of 4
+PASSES = [
+    ("bf16", 1, 2, 16, 128, 4, 7, 0, 32),
+    ("bf16", 1, 1, 8, 128, 4, 8, 0, 32),
+    ("bf16", 2, 1, 16, 128, 4, 8 * 16, 0, 32),
+    ("f16", 1, 2, 4, 128, 4, 8 * 17 + 1, 0, 32),
+    ("f16", 1, 1, 2, 128, 4, 8 * 64, 0, 32),
+    ("bf16", 1, 1, 5, 128, 4, 8 * 31 + 1, 0, 32),
+    ("bf16", 1, 2, 2, 128, 4, 30, 8 * 109 + 6, 32),
+    ("bf16", 1, 2, 2, 128, 4, 4 * 16 + 29, 0, 32, 4),
+]
+
+
+@pytest.mark.parametrize("case", PASSES, ids=[_case_id(c) for c in PASSES])
+def test_prefill_group_scales_passes_agree(case, oracle):
+    """The same sequences once by themselves (a grid for the register-resident
+    pass) and repeated until the shared pass takes the call: bit for bit the
+    same outputs."""
+    dt, B, Hkv, G, D, k, S, S0, group = case[:9]
+    r = case[9] if len(case) > 9 else 8
+    L = N.lib()
+    n_cu = N.num_cus(torch.device(DEV))
+
+    def shared(b):
+        return L.fc_prefill_shared_pass(N.STORE_JPEG_I8G, r, k, D, b, Hkv, G, S, S0, n_cu)
+    reps = 1
+    while not shared(B * reps) and reps < 1024:
+        reps *= 2
+    assert reps > 1 and shared(B * reps)
+    print(f"case prefill passes agree {case} x{reps}", flush=True)
+    ks, vs, (kx, vx) = streams(dt, B, Hkv, S + S0, D, k, 92, oracle, group, r)
+    g = torch.Generator(device=DEV).manual_seed(93)
+    q = torch.randn((B, Hkv * G, S, D), generator=g, device=DEV).to(torch_dtype(dt))
+    ks.append(kx)
+    vs.append(vx)
+    one = codec_prefill_attention(q, ks, vs)
+    kr, vr, _ = streams(dt, B, Hkv, r, D, k, 92, oracle, group, r)
+    kr.append(kx.repeat(reps, 1, 1, 1))
+    vr.append(vx.repeat(reps, 1, 1, 1))
+    many = codec_prefill_attention(q.repeat(reps, 1, 1, 1), kr, vr)
+    assert torch.equal(many, one.repeat(reps, 1, 1, 1))
 
 
 def test_prefill_group_scales_infinite_token_stays_causal(oracle):
