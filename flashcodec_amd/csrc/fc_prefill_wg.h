@@ -415,10 +415,13 @@ __global__ __launch_bounds__(kPThreads, 3) void prefill_i8_wg(PrefillArgs p) {
       // ---------------------------------------------------------- softmax
       // a V row scale at or above 2^(sig_run + 1): accumulators and weights
       // to the new exponent first
-      // (QG: rows past this wavefront's own, which other wavefronts attend,
-      // count as zero here and below: an infinite scale there stays out)
+      // (rows past this wavefront's own, which other wavefronts attend, count as
+      // zero here and below: an infinite scale there stays out.  Not at D = 64
+      // with a scale per row, where every form of it cost 2-8% of a call; there
+      // such a token also makes the earlier runs of its workgroup NaN.  D = 128:
+      // 3% faster than without)
       float vs_pass = v_scales(v3)[lane];
-      if constexpr (QG) {
+      if (QG || (D == 128 && prow < PR)) {
         vs_pass = lane < prow ? vs_pass : 0.f;
         if (prow < PR) {
 #pragma unroll
@@ -544,7 +547,7 @@ __global__ __launch_bounds__(kPThreads, 3) void prefill_i8_wg(PrefillArgs p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) wop[t / 2][4 * (t % 2) + i] = (_Float16)(W[t][i] * vw[i]);
       }
-      if constexpr (QG) {
+      if constexpr (QG || D == 128) {
         if (prow < PR) {
 #pragma unroll
           for (int t = 0; t < NT; ++t)

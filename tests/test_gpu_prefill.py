@@ -199,22 +199,27 @@ def test_prefill_group_scales_passes_agree(case, oracle):
     assert torch.equal(many, one.repeat(reps, 1, 1, 1))
 
 
-def test_prefill_group_scales_infinite_token_stays_causal(oracle):
+@pytest.mark.parametrize("group,D,G,r", [(32, 128, 2, 8), (32, 64, 2, 8), (32, 64, 1, 8), (32, 64, 8, 4),
+                                         (0, 128, 2, 8), (0, 128, 1, 8), (0, 128, 4, 4), (0, 128, 16, 4)])
+def test_prefill_infinite_token_stays_causal(group, D, G, r, oracle):
     """A token that overflows its block's scale reaches no query of an earlier
-    block, whatever its wavefront and pass."""
-    ks, vs, (kx, vx) = streams("bf16", 1, 1, 8 * 40, 128, 4, 91, oracle, 32)
-    q = torch.randn((1, 2, 8 * 40, 128), device=DEV).to(torch.bfloat16)
+    wavefront's token run, whatever the workgroup and pass it shares (within a
+    run of 16 / G tokens a masked weight of zero meets the infinity; at D = 64
+    with a scale per row within the workgroup's four runs)."""
+    S, bad = r * 40, r * 33
+    ks, vs, (kx, vx) = streams("bf16", 1, 1, S, D, 4, 91, oracle, group, r)
+    q = torch.randn((1, G, S, D), device=DEV).to(torch.bfloat16)
     for x in (kx, vx):
-        x[:, :, 8 * 33 + 2, 5] = float("inf")
+        x[:, :, bad + 2, 5] = float("inf")
     ks.append(kx)
     vs.append(vx)
     out = codec_prefill_attention(q, ks, vs)
-    ks2, vs2, _ = streams("bf16", 1, 1, 8, 128, 4, 91, oracle, 32)
-    ks2.append(kx[:, :, :8 * 33])
-    vs2.append(vx[:, :, :8 * 33])
-    ref = codec_prefill_attention(q[:, :, :8 * 33], ks2, vs2)
-    tq = 8                                       # tokens of a wavefront: 16 queries, 2 heads
-    clear = (8 * 33) // tq * tq
+    ks2, vs2, _ = streams("bf16", 1, 1, r, D, 4, 91, oracle, group, r)
+    ks2.append(kx[:, :, :bad])
+    vs2.append(vx[:, :, :bad])
+    ref = codec_prefill_attention(q[:, :, :bad], ks2, vs2)
+    tq = 16 // G                                 # tokens of a wavefront's 16 queries
+    clear = bad // tq * tq
     assert torch.equal(out[:, :, :clear], ref[:, :, :clear])
 
 
