@@ -276,7 +276,9 @@ def _step_args(ks, vs, query, tokens):
     B, Hq, _, D = query.shape
     Hkv = tokens.shape[1]
     dev = query.device
-    key = (id(vs), B, Hq, Hkv, D, query.dtype, ks.dtype, dev)
+    L = N.lib()
+    # (the workspace follows the selected pass's split count)
+    key = (id(vs), B, Hq, Hkv, D, query.dtype, ks.dtype, dev, L.fc_get_attention_pass())
     if plan is not None and plan[0] == key:
         return plan[1], plan[2]
     c = ks.codec
@@ -294,7 +296,6 @@ def _step_args(ks, vs, query, tokens):
     a.r = r
     a.A = _device_A(c, r, dev).data_ptr()
     a.n_cu = N.num_cus(dev)
-    L = N.lib()
     most = L.fc_attention_splits(a.store_kind, a.stream_dtype, a.q_dtype, a.s, 1 << 40, B, Hkv,
                                  Hq // Hkv, D, a.n_cu)
     ws_bytes = L.fc_attention_workspace_bytes(B, Hq, D, most)

@@ -598,3 +598,20 @@ def test_fp_coefficient_widths_infinite_values(dt, D, k, oracle, attention_pass)
     ref = fc.codec_decode_attention(q, ks, vs).float()
     assert int(ref.isinf().sum()) == 2 * B * Hkv * G and not ref.isnan().any()
     assert torch.equal(out.isinf() * out.sign(), ref.isinf() * ref.sign()) and not out.isnan().any()
+
+
+def test_step_plan_follows_the_selected_pass(oracle, attention_pass):
+    """Steps of the same streams under one pass, then the other, which asks
+    for more splits and so for a larger workspace."""
+    B, Hkv, G, D, r, dt = 1, 4, 4, 256, 8, "bf16"
+    print("case step plan under both passes", flush=True)
+    ks, vs = build_streams(dict(mode="jpeg", block_size=r, keep_freqs=1), dt, B, Hkv, r * 4100, D,
+                           181, oracle)
+    torch.cuda.synchronize()
+    fa._WORKSPACES.clear()                  # no larger one of an earlier call
+    g = torch.Generator(device=DEV).manual_seed(182)
+    for name in ("auto", "valu", "auto"):
+        attention_pass(name)
+        q = _tokens(g, B, Hkv * G, D, dt)
+        out = fc.codec_decode_step(q, _tokens(g, B, Hkv, D, dt), _tokens(g, B, Hkv, D, dt), ks, vs)
+        assert_close(to_values(out)[:, :, 0], oracle_out(oracle, q, ks, vs, D ** -0.5), dt)
