@@ -1530,16 +1530,25 @@ int decode_attention_state(const void* q, int q_dtype, int64_t q_sb, int64_t q_s
       (!key->anchors || !value->anchors || !key->masks || !value->masks || s >= r))
     return FC_ERR_ARG;
   const int64_t G = Hq / Hkv;
-  const int n_splits =
+  int n_splits =
       fc_attention_splits(store_kind, stream_dtype, q_dtype, s, nb_hint, B, Hkv, G, D, n_cu);
   if (n_splits < 1) return FC_ERR_UNSUPPORTED;
+  const int64_t mstride = counter_stride(2 * B * Hkv * ((G + 15) / 16));
+  // fp coefficients: no more splits than the fused merge takes (few kv heads and
+  // a long context: 2 heads, D = 256, k = 4, 131072 tokens, 64 splits 55 us, the
+  // vector-ALU pass 124 with its 256 splits, 153 with the 128 sized for the
+  // matrix cores)
+  const bool fpj =
+      store_kind == FC_STORE_JPEG_FP &&
+      split_fpj_mfma_supported(q, q_dtype, q_sb, q_sh, D, s, stream_dtype, key, value) &&
+      mfma_split_allowed() && mstride > 0;
+  if (fpj) n_splits = std::min(n_splits, kFuseMaxSplitsPk);
   if (fc_attention_workspace_bytes(B, Hq, D, n_splits) > workspace_bytes) return FC_ERR_ARG;
   const WsLayout ws = ws_layout(workspace, B, Hq, n_splits);
   unsigned int* counters = ws.counters;
   float* pm = ws.pm;
   float* pl = ws.pl;
   float* pacc = ws.pacc;
-  const int64_t mstride = counter_stride(2 * B * Hkv * ((G + 15) / 16));
   hipStream_t st = (hipStream_t)stream;
   // the same pass fc_attention_splits sized: matrix cores for int8 jpeg
   // archives they support, else the vector-ALU pass; both with the merge
@@ -1587,9 +1596,7 @@ int decode_attention_state(const void* q, int q_dtype, int64_t q_sb, int64_t q_s
                                  scale * kLog2e, pm, pl, pacc, n_splits, counters, kCounterWords,
                                  mstride, &fz, state, st);
   }
-  if (store_kind == FC_STORE_JPEG_FP &&
-      split_fpj_mfma_supported(q, q_dtype, q_sb, q_sh, D, s, stream_dtype, key, value) &&
-      mfma_split_allowed() && mstride > 0 && split_i8_mfma_fusable(n_splits)) {
+  if (fpj) {
     MfmaFuse fz{};
     fz.raw_dtype = stream_dtype;
     fz.n_raw = 0;  // taken from the state

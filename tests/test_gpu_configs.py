@@ -600,6 +600,27 @@ def test_fp_coefficient_widths_infinite_values(dt, D, k, oracle, attention_pass)
     assert torch.equal(out.isinf() * out.sign(), ref.isinf() * ref.sign()) and not out.isnan().any()
 
 
+@pytest.mark.parametrize("dt,r,k,G,D,S,single", [
+    ("bf16", 8, 4, 4, 96, 8 * 40 + 5, True), ("f16", 8, 2, 2, 80, 8 * 33 + 6, True),
+    ("bf16", 8, 2, 8, 256, 8 * 70 + 4, True),
+    # the step's rows exceed its LDS scratch: the multi-launch step
+    ("f16", 16, 4, 4, 256, 16 * 21 + 13, False),
+    # more splits than the fused merge takes: the attention with as many as it does
+    ("bf16", 8, 8, 4, 96, 8 * 2700 + 5, False), ("f16", 16, 8, 2, 256, 16 * 2700 + 13, False),
+])
+def test_fp_coefficient_widths_graph_steps(dt, r, k, G, D, S, single, oracle):
+    """Graph-replayed device-state steps at D = 80, 96, 256 across a block
+    boundary: outputs against the oracle, archives against two appends'."""
+    Hkv = 2
+    print(f"case fp widths graph steps {dt} r={r} k={k} G={G} D={D} S={S}", flush=True)
+    ns = N.lib().fc_attention_splits(N.STORE_JPEG_FP, N.BF16 if dt == "bf16" else N.F16,
+                                     N.BF16 if dt == "bf16" else N.F16, k, S // r, 1, Hkv, G, D,
+                                     N.num_cus(torch.device(DEV)))
+    assert (ns > 64) == (S > 20000), ns
+    _graph_steps(dict(mode="jpeg", block_size=r, keep_freqs=k), dt, 1, Hkv, G, D, S, 5, 171, oracle,
+                 check_archive=True, single_launch=single)
+
+
 def test_step_plan_follows_the_selected_pass(oracle, attention_pass):
     """Steps of the same streams under one pass, then the other, which asks
     for more splits and so for a larger workspace."""
