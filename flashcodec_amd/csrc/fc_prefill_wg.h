@@ -19,10 +19,12 @@
 // the row's largest (rounded to f16), multiplied once per workgroup as the tile
 // is stored, so the ratios are needed one pass before the row scales: the V
 // scales are loaded a pass ahead of their codes.  Bound by the vector ALU and
-// the matrix cores together.  Against the register-resident pass (V converted
-// by every wavefront, masked 64-feature products, 2 wavefronts per SIMD):
-// the last 1000 of 9192 tokens, 2 x 32 heads, D = 128, bf16: 497 -> 431 us (415 us
-// without the selects that keep other wavefronts' rows out).
+// the matrix cores in turn (busy 53% and 28% of the call below, whose 1008
+// workgroups are 1.3 rounds of 768; one scale per row, many rounds: 62% and 38%).
+// Against the register-resident pass (V converted by every wavefront, masked
+// 64-feature products, 2 wavefronts per SIMD): the last 1000 of 9192 tokens, 2 x
+// 32 heads, D = 128, bf16: 501 -> 434 us (3% less without the selects that keep
+// other wavefronts' rows out).  Small grids keep that pass (fc_prefill.hip).
 // The LDS tiles are XOR-swizzled by 16-byte chunk so that the 16
 // lanes of an operand read hit distinct banks.
 #pragma once
